@@ -92,9 +92,8 @@ constexpr KernelMeta pp(int D, int BN, int rings, int dtype, int causal) {
 constexpr KernelMeta kKernelMeta[] = {
     FA_DMA4(128, 64, 2),
     FA_PP4(128, 64, 4),
-    // D = 128, 32-key tiles: the non-causal default, at three workgroups per
-    // CU (1.5-3.7% faster than two, and equal to or up to 3.3% faster than
-    // 64-key tiles at two); the causal kernel spills at three and keeps two.
+    // D = 128, 32-key tiles: non-causal at three workgroups per CU (1.5-3.7%
+    // faster than two); the causal kernel spills at three and keeps two.
     dma(128, 32, 3, FA_DTYPE_FP16, 0), dma(128, 32, 2, FA_DTYPE_FP16, 1),
     dma(128, 32, 3, FA_DTYPE_BF16, 0), dma(128, 32, 2, FA_DTYPE_BF16, 1),
     // D <= 64 is softmax (VALU) bound, and a single wave issues VALU work
@@ -139,15 +138,20 @@ constexpr bool table_fits_lds() {
 static_assert(table_fits_lds(), "LDS budget of one gfx950 CU");
 
 // Default (BLOCK_N, waves) per head dim; BLOCK_M = 32 * waves.
-void default_tiling(int D, int dtype, int causal, int *bn, int *nw) {
+void default_tiling(int D, int dtype, int *bn, int *nw) {
   // fp8 V: 64-key tiles (D = 16: 128), one 32x32x64 MFMA per 64 keys and 32
-  // head dims.  16-bit V: 64 keys, except D = 16 (128), D = 256 (32) and
-  // non-causal D = 128 (32, the three-workgroups-per-CU kernel).
+  // head dims.  16-bit V: 64 keys, except D = 16 (128) and D = 256 (32).
+  // Non-causal D = 128 took the 32-key kernel (three workgroups per CU) before
+  // the 64-key one carried its tile as two 32-key blocks; over grids of 8 to
+  // 1536 tiles and 256 to 8192 keys the 64-key kernel is now the faster on
+  // every one, by 3-9% on full grids and 13-25% up to one tile per CU (fp16,
+  // us, 32 against 64 keys: H16 S2048 43.5 / 37.9, H32 S4096 270 / 258,
+  // H16 S1024 22.9 / 18.3).
   if (v_is_fp8(dtype))
     *bn = D == 16 ? 128 : 64;
   else if (D == 16)
     *bn = 128;
-  else if (D == 256 || (D == 128 && !causal))
+  else if (D == 256)
     *bn = 32;
   else
     *bn = 64;
@@ -179,7 +183,7 @@ constexpr int kDefaultCuCount = 256;
 int make_plan(const fa_fwd_params *p, Plan *out, int cu_count = kDefaultCuCount, int splits = 1) {
   int bn, nw;
   if (p->block_m == 0 && p->block_n == 0) {
-    default_tiling(p->D, p->dtype, p->causal, &bn, &nw);
+    default_tiling(p->D, p->dtype, &bn, &nw);
   } else {
     if (p->block_m <= 0 || p->block_n <= 0 || p->block_m % 32 != 0) return FA_ERR_TILING;
     bn = p->block_n;
