@@ -202,7 +202,11 @@ __device__ __forceinline__ int vt_pos(int k) {
 // once) that pulls (head, m-tile) tiles from nq = min(8, grid, B*H) queues:
 // workgroup b serves queue b % nq (the dispatcher sends workgroup b to XCD
 // b % 8, so a queue is an XCD's), and queue x owns heads x, x+nq, x+2nq, ...,
-// so a head's K/V is only ever read through one XCD's L2.  A queue hands out
+// so a head's K/V is only ever read through one XCD's L2.  B*H mod nq heads
+// are left over; their tiles are dealt to all queues in turn.  As whole heads
+// on some of the queues, they kept those queues' workgroups busy while the
+// others' had nothing left (fp16, us: H12 S2048 D128 57.6 -> 32.2, D64 44.2 ->
+// 23.7; H20 S4096 D128 causal 110 -> 99).  A queue hands out
 // its tiles heaviest first (causal: largest m-tile first, across its heads),
 // so the tail is made of the cheapest tiles.  Pulling instead of a static
 // split matters on gfx950: workgroups sharing a CU do not progress at the
@@ -235,14 +239,18 @@ struct TileQueue {
   uint32_t n_tiles;   // tiles of this queue
   uint32_t n_static;  // tickets taken without the counter: min(workers, n_tiles)
   uint32_t workers;   // workgroups serving this queue
-  int x, nq, nh;      // queue index, queue count, heads of this queue
+  uint32_t n_extra;   // tiles of the left-over heads that this queue takes, per KV split
+  int x, nq, nh;      // queue index, queue count, whole heads of this queue
+  int n_left;         // left-over heads: nq * nh .. B * H - 1
 
   __device__ __forceinline__ TileQueue(const KernelArgs &p) {
     nq = p.nq;
     x = blockIdx.x % nq;
     const int BH = p.B * p.H;
-    nh = (BH - x + nq - 1) / nq;
-    n_tiles = (uint32_t)nh * (uint32_t)p.n_mtiles * (uint32_t)p.kv_splits;
+    nh = BH / nq;
+    n_left = BH - nh * nq;
+    n_extra = ((uint32_t)n_left * (uint32_t)p.n_mtiles + (uint32_t)(nq - 1 - x)) / (uint32_t)nq;
+    n_tiles = ((uint32_t)nh * (uint32_t)p.n_mtiles + n_extra) * (uint32_t)p.kv_splits;
     workers = (gridDim.x - x + nq - 1) / nq;
     n_static = workers < n_tiles ? workers : n_tiles;
     ctr = p.queue != nullptr ? p.queue + x * kQueueStride : nullptr;
@@ -260,7 +268,8 @@ struct TileQueue {
   }
   // Ticket -> (head bh, m-tile mt, KV split); false past the end.  Order:
   // KV splits one after the other (split 0 holds the most work); inside a
-  // split, the weight ranks k (0 = heaviest m-tile) are cut into `bands`
+  // split, this queue's share of the left-over heads (rank-major), then its
+  // own heads: the weight ranks k (0 = heaviest m-tile) are cut into `bands`
   // bands; band by band, the queue's heads go in groups of `group`, and
   // inside a group rank-major (heaviest first across the group's heads).
   // Small groups keep a group's K/V in the XCD's L2; bands bound how heavy
@@ -268,9 +277,17 @@ struct TileQueue {
   __device__ __forceinline__ bool tile(uint32_t t, int n_mtiles, bool causal, int group, int bands,
                                        int *bh, int *mt, int *split) const {
     if (t >= n_tiles) return false;
-    const uint32_t per_split = (uint32_t)nh * (uint32_t)n_mtiles;
+    const uint32_t per_split = (uint32_t)nh * (uint32_t)n_mtiles + n_extra;
     *split = (int)(t / per_split);
     t -= (uint32_t)*split * per_split;
+    if (t < n_extra) {
+      const uint32_t e = (uint32_t)x + (uint32_t)nq * t;
+      const uint32_t ke = e / (uint32_t)n_left;
+      *bh = nq * nh + (int)(e - ke * (uint32_t)n_left);
+      *mt = causal ? n_mtiles - 1 - (int)ke : (int)ke;
+      return true;
+    }
+    t -= n_extra;
     const int bs = (n_mtiles + bands - 1) / bands;     // ranks per band
     const uint32_t per_band = (uint32_t)nh * (uint32_t)bs;
     const int b = (int)(t / per_band);
