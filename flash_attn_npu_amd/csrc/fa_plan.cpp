@@ -359,26 +359,40 @@ int32_t fa_default_kv_splits(const fa_fwd_params *p) {
   if (make_plan(p, &plan) != FA_OK) return 1;
   const KernelMeta &e = kKernelMeta[plan.kernel];
   if (!e.splittable) return 1;
-  // Fitted to 25 shapes timed on MI355X with 1..8 splits (B1-2, H1-16,
-  // S256-16384, D16-256, fp16):
-  //  * only grids of at most half a workgroup per CU split: at one tile per
-  //    CU (256) a second workgroup per CU gained nothing (B1 H8 S4096 D64:
-  //    50 -> 54 us with 2 splits) or at most 3-5%;
-  //  * the runs fill one workgroup per CU, two for causal grids, whose
-  //    longest m-tile (all keys) sets the time while the others finish
-  //    early (B1 H4 S4096 D128 causal: 62 -> 42 us at 2, 41 at 4);
-  //  * each run keeps at least 64K key-columns (Sk / splits * D >= 65536):
-  //    below that the merge launch and its HBM pass cost more than the
-  //    shorter runs save (B1 H4 S1024 D64: 14.7 -> 15.7 us at 2 splits).
-  // These picks were within 8% of the fastest split count on every shape
-  // timed (18 of 25 the fastest), against up to 18% slower under the earlier
-  // rule (at least 8 KV tiles and 512 keys a run, up to two workgroups per CU).
-  if (plan.total_tiles * 2 > kDefaultCuCount) return 1;
-  const int64_t fill = (p->causal ? 2 : 1) * kDefaultCuCount / plan.total_tiles;
-  const int64_t work = (int64_t)p->Sk * p->D / 65536;
-  int64_t splits = fill < work ? fill : work;
-  if (splits > kMaxKvSplits) splits = kMaxKvSplits;
-  return splits > 1 ? (int32_t)splits : 1;
+  // A grid of at most one tile per CU takes as long as one workgroup needs
+  // for all its keys, and splitting them pays what the merge costs: its launch,
+  // and one pass of the partial O (tiles * splits of them) out and in.  Both are
+  // estimated in us from timings over 8 to 256 tiles, 256 to 8192 keys and
+  // every head dim (fp16, 2 to 16 splits); the power of two with the
+  // largest gain wins, or none:
+  //  * a lone workgroup's time per key grows with D (H16 S1024 D128: 18.3 us,
+  //    H8 S2048 29.6, H4 S4096 31.5 at D = 16);
+  //  * the merge costs 5 us, 0.2 per split and 0.03 per tile and split at
+  //    D = 128; causal launches write less, their runs past the diagonal being empty;
+  //  * runs of at least 128 keys, and one workgroup per CU: more only when
+  //    causal, where half of the work is missing, with runs of 2048 keys.
+  // Against the rule before (at least 64K key-columns a run, one workgroup per
+  // CU, two if causal), us: H8 S2048 D16 18.2 -> 15.5, H1 S4096 D32 23.4 ->
+  // 16.6, H2 S2048 D64 18.0 -> 16.4, H16 S1024 D128 26.2 -> 18.3, H16 S1024
+  // D256 causal 51.9 -> 31.2; over that sweep it is within 1% of the fastest
+  // choice on average (3.6% before).
+  if (plan.total_tiles > kDefaultCuCount) return 1;
+  const double key_us = (p->D == 16 ? 6.5 : p->D == 32 ? 7.5 : p->D == 64 ? 9.3 : p->D == 128 ? 11.7 : 23.0) / 1024;
+  const double tile_us = 0.030 * (p->causal ? 0.6 : 1.0) * p->D / 128;
+  double best = 0.0;
+  int splits = 1;
+  for (int s = 2; s <= kMaxKvSplits; s *= 2) {
+    const int64_t run = p->Sk / s, groups = plan.total_tiles * s;
+    int64_t limit = kDefaultCuCount;
+    if (p->causal && run >= 2048) limit = plan.total_tiles <= kDefaultCuCount / 2 && p->D <= 128 ? 512 : 384;
+    if (run < 128 || groups > limit) break;
+    const double gain = p->Sk * key_us * (1.0 - 1.0 / s) - (5.0 + 0.2 * s + tile_us * (double)groups);
+    if (gain > best) {
+      best = gain;
+      splits = s;
+    }
+  }
+  return splits;
 }
 
 }  // extern "C"

@@ -178,10 +178,9 @@ int64_t fa_split_workspace_bytes(const fa_fwd_params *p, int32_t kv_splits);
 int fa_fwd_split(const fa_fwd_params *p, int32_t kv_splits, void *workspace, int64_t workspace_bytes,
                  void *hip_stream);
 
-/* The library's split choice for these parameters: > 1 only when the
- * unsplit grid has at most one (head, m-tile) tile per two CUs; the runs then
- * fill one workgroup per CU (two for a causal mask), each keeping at least
- * 65536 key-columns (Sk / splits * D).  Host-only. */
+/* The library's split choice for these parameters: > 1 only when the unsplit
+ * grid has at most one (head, m-tile) tile per CU and the shorter runs are
+ * estimated to save more than the merge costs.  Host-only. */
 int32_t fa_default_kv_splits(const fa_fwd_params *p);
 
 /* ---- No-allocation split-KV.  No counterpart in the reference.  For callers

@@ -16,3 +16,28 @@ def test_default_tile_follows_head_dim(head_dim, block_n, causal, dtype):
         rt = fa._describe_runtime(3, 5, n_ctx, head_dim, causal, dtype=dtype)
         assert rt["tiling_source"] == "fallback"
         assert rt["selected_config"] == {"BLOCK_M": 128, "BLOCK_N": block_n}
+
+
+def _splits(z, h, n_ctx, head_dim, causal):
+    return fa._describe_runtime(z, h, n_ctx, head_dim, causal)["kv_splits"]
+
+
+def test_split_choice_at_its_limits():
+    # 128 tiles of 1024 keys: the merge would cost more than the halved runs save.
+    assert _splits(1, 16, 1024, 128, False) == 1
+    assert _splits(1, 16, 1024, 256, True) == 1
+    # 128 tiles of 4096 keys: two runs fill the CUs.
+    assert _splits(1, 4, 4096, 128, False) == 2
+    assert _splits(1, 8, 2048, 16, False) == 2
+    # One tile per CU and more: none.
+    assert _splits(1, 8, 4096, 64, False) == 1
+    assert _splits(1, 8, 4096, 64, True) == 1
+    assert _splits(1, 9, 4096, 64, False) == 1
+    # 192 tiles: causal runs may share CUs when they are long, others not.
+    assert _splits(1, 3, 8192, 64, True) == 2
+    assert _splits(1, 3, 8192, 64, False) == 1
+    # Short runs are never made.
+    assert _splits(1, 1, 128, 256, False) == 1
+    for n_ctx in (129, 300, 1000, 4097, 100000):
+        s = _splits(1, 1, n_ctx, 128, False)
+        assert s == 1 or (n_ctx // s >= 128 and s * -(-n_ctx // 128) <= 256)
