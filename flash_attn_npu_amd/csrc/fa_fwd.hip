@@ -40,8 +40,9 @@
 //  * Grid: persistent (as many workgroups as are resident at once); the
 //    workgroups of each XCD pull (head, m-tile) tiles, heaviest first, from
 //    a tile queue that owns a fixed set of heads, so a head's K/V is read
-//    through one L2.  Grids too small to fill the chip split the keys
-//    (split-KV) and merge the partial results in a second kernel.
+//    through one L2 (heads left over are dealt to all queues).  Grids too
+//    small to fill the chip split the keys (split-KV) and merge the partial
+//    results in a second kernel.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -101,12 +102,8 @@ struct KernelArgs {
   int64_t v_sb, v_sh, v_ss;
   int64_t o_sb, o_sh, o_ss;
   int32_t B, H, Sq, Sk;
-  int32_t n_mtiles;     // ceil(Sq / BM)
-  int32_t total_tiles;  // n_mtiles * B * H
   unsigned long long *queue;  // this launch's tile-queue counters (see TileQueue)
-  int32_t nq;                 // tile queues: min(8, grid, B*H)
-  int32_t q_group;            // heads per group in a queue's order (>= 1)
-  int32_t q_bands;            // weight bands in a queue's order (>= 1)
+  TileOrder order;            // units of the queues
   // Split-KV (DMA kernel only): kv_splits > 1 cuts every m-tile's KV range
   // into runs of split_tiles tiles; each run writes a partial O (fp32,
   // normalised by its own row sum) and its natural-log LSE, and
@@ -201,32 +198,31 @@ __device__ __forceinline__ int vt_pos(int k) {
 // Every kernel runs a persistent grid (as many workgroups as are resident at
 // once) that pulls (head, m-tile) tiles from nq = min(8, grid, B*H) queues:
 // workgroup b serves queue b % nq (the dispatcher sends workgroup b to XCD
-// b % 8, so a queue is an XCD's), and queue x owns heads x, x+nq, x+2nq, ...,
-// so a head's K/V is only ever read through one XCD's L2.  B*H mod nq heads
-// are left over; their tiles are dealt to all queues in turn.  As whole heads
+// b % 8, so a queue is an XCD's), and a queue owns every nq-th head, so a
+// head's K/V is only read through one XCD's L2, but for the B*H mod nq
+// left-over heads, whose tiles are dealt to all queues in turn.  As whole heads
 // on some of the queues, they kept those queues' workgroups busy while the
-// others' had nothing left (fp16, us: H12 S2048 D128 57.6 -> 32.2, D64 44.2 ->
-// 23.7; H20 S4096 D128 causal 110 -> 99).  A queue hands out
-// its tiles heaviest first (causal: largest m-tile first, across its heads),
+// others' had nothing left (fp16, us: H12 S2048 D128 59 -> 33, D64 45 -> 24;
+// H28 S4096 D128 causal 131 -> 117).  TileOrder (fa_plan.cpp) is the order
+// in which a queue hands out its tiles, heaviest first inside a group of heads,
 // so the tail is made of the cheapest tiles.  Pulling instead of a static
 // split matters on gfx950: workgroups sharing a CU do not progress at the
 // same rate (the older one wins issue arbitration), so any fixed assignment
 // leaves some of them idle at the end.
 //
-// Ticket i of a queue is its i-th heaviest tile.  The queue's W workgroups
-// take tickets 0..W-1 statically (no atomic before the first tile); later
-// tickets come from a counter: ticket = W + atomicAdd(counter, 1), requested
-// at the top of a tile so its latency hides behind the tile.  Each of those
-// workgroups takes exactly one ticket past the end and stops, so the taker of
-// raw count n_tiles - 1 is the last user of the counter and resets it to 0:
-// the next launch finds it clean.  The counters live in a device array owned
-// by the library, one group of kQueues per launch slot (one 128-byte line per
-// counter); launch slots rotate over kQueueSlots, which bounds the eager
-// launches that may be in flight on one device.
+// The queue's W workgroups take tickets 0..W-1 statically (no atomic before
+// the first tile); later tickets come from a counter: ticket = W +
+// atomicAdd(counter, 1), requested at the top of a tile so its latency hides
+// behind the tile.  Each of those workgroups takes exactly one ticket past the
+// end and stops, so the taker of raw count n_tiles - 1 is the last user of the
+// counter and resets it to 0: the next launch finds it clean.  The counters
+// live in a device array owned by the library, one group of kQueues per launch
+// slot (one 128-byte line per counter); launch slots rotate over kQueueSlots,
+// which bounds the eager launches that may be in flight on one device.
 //
 // A launch recorded into a graph (its stream is capturing) gets no counters
-// (KernelArgs::queue == nullptr): its workgroups walk the same heaviest-first
-// ticket order statically, workgroup w of a queue taking tickets w, w + W,
+// (KernelArgs::queue == nullptr): its workgroups walk the same ticket order
+// statically, workgroup w of a queue taking tickets w, w + W,
 // w + 2W, ...  Replays of captured launches therefore share no device state
 // with each other or with eager launches, whatever streams they run on.
 constexpr int kQueues = 8;
@@ -239,18 +235,12 @@ struct TileQueue {
   uint32_t n_tiles;   // tiles of this queue
   uint32_t n_static;  // tickets taken without the counter: min(workers, n_tiles)
   uint32_t workers;   // workgroups serving this queue
-  uint32_t n_extra;   // tiles of the left-over heads that this queue takes, per KV split
-  int x, nq, nh;      // queue index, queue count, whole heads of this queue
-  int n_left;         // left-over heads: nq * nh .. B * H - 1
+  int x, nq;          // queue index, queue count
 
   __device__ __forceinline__ TileQueue(const KernelArgs &p) {
-    nq = p.nq;
+    nq = p.order.nq;
     x = blockIdx.x % nq;
-    const int BH = p.B * p.H;
-    nh = BH / nq;
-    n_left = BH - nh * nq;
-    n_extra = ((uint32_t)n_left * (uint32_t)p.n_mtiles + (uint32_t)(nq - 1 - x)) / (uint32_t)nq;
-    n_tiles = ((uint32_t)nh * (uint32_t)p.n_mtiles + n_extra) * (uint32_t)p.kv_splits;
+    n_tiles = queue_tickets(p.order, x);
     workers = (gridDim.x - x + nq - 1) / nq;
     n_static = workers < n_tiles ? workers : n_tiles;
     ctr = p.queue != nullptr ? p.queue + x * kQueueStride : nullptr;
@@ -266,42 +256,13 @@ struct TileQueue {
     if (raw == n_tiles - 1) atomicExch(ctr, 0ull);
     return n_static + (uint32_t)raw;
   }
-  // Ticket -> (head bh, m-tile mt, KV split); false past the end.  Order:
-  // KV splits one after the other (split 0 holds the most work); inside a
-  // split, this queue's share of the left-over heads (rank-major), then its
-  // own heads: the weight ranks k (0 = heaviest m-tile) are cut into `bands`
-  // bands; band by band, the queue's heads go in groups of `group`, and
-  // inside a group rank-major (heaviest first across the group's heads).
-  // Small groups keep a group's K/V in the XCD's L2; bands bound how heavy
-  // the last group's tiles are.
-  __device__ __forceinline__ bool tile(uint32_t t, int n_mtiles, bool causal, int group, int bands,
-                                       int *bh, int *mt, int *split) const {
+  // Ticket -> (head bh, m-tile mt, KV split); false past the end.  The host works
+  // out the order's constants (one division and three values fewer live through a
+  // unit than with the device's: 1-2% on the shortest launches, 1% on the rest).
+  __device__ __forceinline__ bool tile(const KernelArgs &p, uint32_t t, bool causal, int *bh, int *mt,
+                                       int *split) const {
     if (t >= n_tiles) return false;
-    const uint32_t per_split = (uint32_t)nh * (uint32_t)n_mtiles + n_extra;
-    *split = (int)(t / per_split);
-    t -= (uint32_t)*split * per_split;
-    if (t < n_extra) {
-      const uint32_t e = (uint32_t)x + (uint32_t)nq * t;
-      const uint32_t ke = e / (uint32_t)n_left;
-      *bh = nq * nh + (int)(e - ke * (uint32_t)n_left);
-      *mt = causal ? n_mtiles - 1 - (int)ke : (int)ke;
-      return true;
-    }
-    t -= n_extra;
-    const int bs = (n_mtiles + bands - 1) / bands;     // ranks per band
-    const uint32_t per_band = (uint32_t)nh * (uint32_t)bs;
-    const int b = (int)(t / per_band);
-    const uint32_t r = t - (uint32_t)b * per_band;
-    const int len = min(bs, n_mtiles - b * bs);          // ranks in this band
-    const uint32_t per_group = (uint32_t)group * (uint32_t)len;
-    const int g = (int)(r / per_group);
-    const uint32_t r2 = r - (uint32_t)g * per_group;
-    const int gsz = min(group, nh - g * group);          // heads in this group
-    const int kk = (int)(r2 / (uint32_t)gsz);
-    const int hi = (int)(r2 - (uint32_t)kk * gsz);
-    const int k = b * bs + kk;
-    *bh = x + nq * (g * group + hi);
-    *mt = causal ? n_mtiles - 1 - k : k;
+    tile_of_ticket(p.order, x, t, causal, bh, mt, split);
     return true;
   }
 };
@@ -576,9 +537,7 @@ fa_fwd_dma_kernel(KernelArgs p) {
   __shared__ uint32_t s_ticket[2];
   const TileQueue tq(p);
   int bh, mt, split;
-  for (int it = 0; tq.tile(it == 0 ? tq.first() : s_ticket[it & 1], p.n_mtiles, CAUSAL, p.q_group, p.q_bands,
-                           &bh, &mt, &split);
-       ++it) {
+  for (int it = 0; tq.tile(p, it == 0 ? tq.first() : s_ticket[it & 1], CAUSAL, &bh, &mt, &split); ++it) {
     unsigned long long next_raw = 0;
 #ifdef FA_TIMING
     uint32_t tm_vm = 0, tm_bar = 0, tm_cmp = 0, n_comp = 0, tm_pro = 0, tm_epi0 = 0, tm_dma = 0, tm_idle = 0;
@@ -1513,9 +1472,7 @@ fa_fwd_pp_kernel(KernelArgs p) {
   __shared__ uint32_t s_ticket[2];
   const TileQueue tq(p);
   int bh, mt, split;
-  for (int it = 0; tq.tile(it == 0 ? tq.first() : s_ticket[it & 1], p.n_mtiles, CAUSAL, p.q_group, p.q_bands,
-                           &bh, &mt, &split);
-       ++it) {
+  for (int it = 0; tq.tile(p, it == 0 ? tq.first() : s_ticket[it & 1], CAUSAL, &bh, &mt, &split); ++it) {
     unsigned long long next_raw = 0;
     if (threadIdx.x == 0) next_raw = tq.request();
 #ifdef FA_TIMING
@@ -2037,8 +1994,6 @@ int launch(const fa_fwd_params *p, void *hip_stream, int splits, void *workspace
   a.H = p->H;
   a.Sq = p->Sq;
   a.Sk = p->Sk;
-  a.n_mtiles = plan.n_mtiles;
-  a.total_tiles = (int32_t)plan.total_tiles;
   a.kv_splits = splits > 1 ? splits : 1;
   a.split_tiles = splits > 1 ? plan.split_tiles : (1 << 30);
   a.part_o = splits > 1 ? (float *)workspace : nullptr;
@@ -2062,17 +2017,7 @@ int launch(const fa_fwd_params *p, void *hip_stream, int splits, void *workspace
     int64_t nq = kQueues;
     if (nq > plan.grid) nq = plan.grid;
     if (nq > bh) nq = bh;
-    a.nq = (int32_t)nq;
-    // Queue order: a queue's heads in groups of 8, each group's tiles
-    // heaviest first across its heads, one band.  Measured on the benchmark
-    // workloads against groups of 2..64 heads and 1..4 bands: within 1% of
-    // the best time on each, with the least HBM traffic or close to it
-    // (e.g. B8 H32 S3000 causal: 646 us and 2.5 GB fetched per launch, against
-    // 804 us and 6.6 GB for all 32 heads of a queue at once; B16 H16 S1024:
-    // 87 us against 101 us).
-    const int64_t nh = (bh + nq - 1) / nq;  // heads of queue 0
-    a.q_group = (int32_t)(nh < 8 ? (nh > 0 ? nh : 1) : 8);
-    a.q_bands = 1;
+    a.order = make_tile_order((int)bh, plan.n_mtiles, a.kv_splits, (int)nq);
   }
   // A negative scale is folded into Q (sign flip of every element, exact),
   // a zero scale into a tiny positive one (all logits ~0: uniform weights).

@@ -214,6 +214,78 @@ int make_plan(const fa_fwd_params *p, Plan *out, int cu_count = kDefaultCuCount,
   return FA_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Order of the persistent grid's work.  A unit is a (head, m-tile, KV run); the
+// units are dealt to nq queues (TileQueue in fa_fwd.hip), and ticket t of queue x
+// is the t-th unit of its list.  Queue x owns heads x, x + nq, x + 2 nq, ..., so a
+// whole head's K/V is read through one queue's L2; it takes them in groups of 8,
+// and inside a group KV run by KV run and m-tile by m-tile, heaviest first
+// (causal: the largest), each through the group's heads.  The B*H mod nq heads
+// left over go with the last group: their tiles are dealt to the queues in turn,
+// each m-tile's after the queue's own heads.  So every list stays heaviest first,
+// and the queues' unit counts differ by at most one, as the workgroups of a grid
+// of one per unit do.  Dealt before everything else, light tiles with heavy
+// ones, the left-over heads made causal B*H = 15 S4096 (fp16) 48 us at D = 32 and
+// 201 at D = 256, against 35 and 165 here and 37 and 173 with whole heads on
+// some of the queues.
+struct TileOrder {
+  int32_t nq;        // queues
+  int32_t n_mtiles;
+  int32_t ranks;     // m-tiles * KV runs
+  int32_t heads;     // B*H
+  int32_t cols;      // heads of a group but the last: nq * heads per queue and group
+  int32_t own;       // where heads are left over: the last group's other heads
+  int32_t last;      // index of the last group
+  int32_t tickets;   // tickets of a queue in a group but the last
+};
+
+constexpr TileOrder make_tile_order(int heads, int n_mtiles, int splits, int nq) {
+  // Groups of 8 heads per queue.  Measured on the benchmark workloads against
+  // groups of 2..64 heads: within 1% of the best time on each, with the
+  // least HBM traffic or close to it (e.g. B8 H32 S3000 causal: 646 us and
+  // 2.5 GB fetched per launch, against 804 us and 6.6 GB for all 32 heads of
+  // a queue at once; B16 H16 S1024: 87 us against 101 us).
+  const int per_queue = heads / nq;  // >= 1
+  const int left = heads % nq;
+  const int group = per_queue < 8 ? per_queue : 8;
+  TileOrder o = {};
+  o.nq = nq;
+  o.n_mtiles = n_mtiles;
+  o.ranks = n_mtiles * splits;
+  o.heads = heads;
+  o.cols = nq * group;
+  o.last = (per_queue - 1) / group;
+  o.tickets = group * o.ranks;
+  // (With fewer than 8 queues, a program count's, the last group's heads all take turns.)
+  o.own = left != 0 && nq == 8 ? heads - left - o.last * o.cols : 0;
+  return o;
+}
+
+// Tickets of queue x.
+__attribute__((always_inline)) constexpr uint32_t queue_tickets(const TileOrder &o, int x) {
+  return ((uint32_t)o.heads * (uint32_t)o.ranks - (uint32_t)x + (uint32_t)o.nq - 1) / (uint32_t)o.nq;
+}
+
+// Ticket t < queue_tickets(o, x) of queue x -> (head, m-tile, KV run): element
+// x + nq * t of the group's list (rank, column), `cols` heads wide.
+__attribute__((always_inline)) constexpr void tile_of_ticket(const TileOrder &o, int x, uint32_t t, bool causal, int *bh,
+                                                             int *mt, int *split) {
+  uint32_t g = t / (uint32_t)o.tickets;
+  if (g > (uint32_t)o.last) g = (uint32_t)o.last;
+  const uint32_t base = g * (uint32_t)o.cols;  // first head of the group
+  const uint32_t cols = g == (uint32_t)o.last ? (uint32_t)o.heads - base : (uint32_t)o.cols;
+  const uint32_t e = (uint32_t)x + (uint32_t)o.nq * (t - g * (uint32_t)o.tickets);
+  const uint32_t rank = e / cols;
+  uint32_t col = e - rank * cols;
+  // Where cols is no multiple of the 8 queues, their turn moves on from rank to
+  // rank; of each block of 8 whole heads, this queue's own is the one to take.
+  if (col < (uint32_t)o.own) col = (col & ~7u) + (uint32_t)x;
+  *bh = (int)(base + col);
+  *split = (int)(rank / (uint32_t)o.n_mtiles);
+  const int k = (int)(rank - (uint32_t)*split * (uint32_t)o.n_mtiles);
+  *mt = causal ? o.n_mtiles - 1 - k : k;
+}
+
 bool aligned16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 // Workspace of a split-KV launch: partial O, then (256-byte aligned) LSE.
