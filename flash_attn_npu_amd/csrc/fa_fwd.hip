@@ -2017,7 +2017,7 @@ int launch(const fa_fwd_params *p, void *hip_stream, int splits, void *workspace
     int64_t nq = kQueues;
     if (nq > plan.grid) nq = plan.grid;
     if (nq > bh) nq = bh;
-    a.order = make_tile_order((int)bh, plan.n_mtiles, a.kv_splits, (int)nq);
+    a.order = make_tile_order((int)bh, plan.n_mtiles, a.kv_splits, (int)nq, p->causal != 0, plan.grid, cu_count);
   }
   // A negative scale is folded into Q (sign flip of every element, exact),
   // a zero scale into a tiny positive one (all logits ~0: uniform weights).

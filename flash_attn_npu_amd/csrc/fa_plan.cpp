@@ -222,24 +222,31 @@ int make_plan(const fa_fwd_params *p, Plan *out, int cu_count = kDefaultCuCount,
 // and inside a group KV run by KV run and m-tile by m-tile, heaviest first
 // (causal: the largest), each through the group's heads.  The B*H mod nq heads
 // left over go with the last group: their tiles are dealt to the queues in turn,
-// each m-tile's after the queue's own heads.  So every list stays heaviest first,
-// and the queues' unit counts differ by at most one, as the workgroups of a grid
-// of one per unit do.  Dealt before everything else, light tiles with heavy
-// ones, the left-over heads made causal B*H = 15 S4096 (fp16) 48 us at D = 32 and
-// 201 at D = 256, against 35 and 165 here and 37 and 173 with whole heads on
-// some of the queues.
+// each m-tile's after the queue's own heads (make_tile_order has one exception).
+// So every list stays heaviest first, and the queues' unit counts differ by at
+// most one, as the workgroups of a grid of one per unit do.  Dealt before
+// everything else, light tiles with heavy ones, the left-over heads made causal
+// B*H = 15 S4096 (fp16) 48 us at D = 32 and 201 at D = 256, against 35 and 165
+// here and 37 and 173 with whole heads on some of the queues.
+//
+// The padding groups what the compiler loads together: the default kernels spill
+// 54-103 scalar registers with it, up to 25 more without.
 struct TileOrder {
   int32_t nq;        // queues
   int32_t n_mtiles;
   int32_t ranks;     // m-tiles * KV runs
-  int32_t heads;     // B*H
+  int32_t heads0;    // queue 0's heads: as below, or, with a whole left-over head, heads + nq
+  int32_t heads;     // B*H; less the left-over head where queue 0 has it whole
+  int32_t pad[2];
   int32_t cols;      // heads of a group but the last: nq * heads per queue and group
   int32_t own;       // where heads are left over: the last group's other heads
   int32_t last;      // index of the last group
   int32_t tickets;   // tickets of a queue in a group but the last
+  int32_t pad2;
 };
 
-constexpr TileOrder make_tile_order(int heads, int n_mtiles, int splits, int nq) {
+// `grid` workgroups on `cu_count` CUs.
+constexpr TileOrder make_tile_order(int heads, int n_mtiles, int splits, int nq, bool causal, int grid, int cu_count) {
   // Groups of 8 heads per queue.  Measured on the benchmark workloads against
   // groups of 2..64 heads: within 1% of the best time on each, with the
   // least HBM traffic or close to it (e.g. B8 H32 S3000 causal: 646 us and
@@ -252,18 +259,31 @@ constexpr TileOrder make_tile_order(int heads, int n_mtiles, int splits, int nq)
   o.nq = nq;
   o.n_mtiles = n_mtiles;
   o.ranks = n_mtiles * splits;
-  o.heads = heads;
   o.cols = nq * group;
   o.last = (per_queue - 1) / group;
   o.tickets = group * o.ranks;
+  // Non-causal, where tiles are all alike: one left-over head stays whole, one
+  // more of queue 0's own, on grids of more units than workgroups where its tiles
+  // cost queue 0's CUs no further round.  Dealt, they make every queue start
+  // one for a few tiles, 1-7% slower (fp16, us, whole / dealt: B*H = 97 S2048
+  // D128 194 / 202, D256 449 / 484, 65 S1024 D128 48 / 50).  Where the whole head
+  // costs a round more, dealt is up to 1.45x faster (9 S8192 D32), on grids of
+  // one round up to 1.8x, and with two heads and more left over 1-7% on average.
+  const int cus = cu_count / nq > 0 ? cu_count / nq : 1;  // of one queue
+  const int64_t dealt = ((int64_t)heads * o.ranks + nq - 1) / nq, whole = (int64_t)(per_queue + 1) * o.ranks;
+  const bool keep = !causal && left == 1 && (int64_t)heads * o.ranks > grid &&
+                    (dealt + cus - 1) / cus == (whole + cus - 1) / cus;
+  o.heads = keep ? heads - 1 : heads;
+  o.heads0 = keep ? heads - 1 + nq : heads;
   // (With fewer than 8 queues, a program count's, the last group's heads all take turns.)
-  o.own = left != 0 && nq == 8 ? heads - left - o.last * o.cols : 0;
+  o.own = left != 0 && !keep && nq == 8 ? heads - left - o.last * o.cols : 0;
   return o;
 }
 
 // Tickets of queue x.
 __attribute__((always_inline)) constexpr uint32_t queue_tickets(const TileOrder &o, int x) {
-  return ((uint32_t)o.heads * (uint32_t)o.ranks - (uint32_t)x + (uint32_t)o.nq - 1) / (uint32_t)o.nq;
+  const uint32_t heads = (uint32_t)(x == 0 ? o.heads0 : o.heads);
+  return (heads * (uint32_t)o.ranks - (uint32_t)x + (uint32_t)o.nq - 1) / (uint32_t)o.nq;
 }
 
 // Ticket t < queue_tickets(o, x) of queue x -> (head, m-tile, KV run): element
@@ -273,7 +293,7 @@ __attribute__((always_inline)) constexpr void tile_of_ticket(const TileOrder &o,
   uint32_t g = t / (uint32_t)o.tickets;
   if (g > (uint32_t)o.last) g = (uint32_t)o.last;
   const uint32_t base = g * (uint32_t)o.cols;  // first head of the group
-  const uint32_t cols = g == (uint32_t)o.last ? (uint32_t)o.heads - base : (uint32_t)o.cols;
+  const uint32_t cols = g == (uint32_t)o.last ? (uint32_t)(x == 0 ? o.heads0 : o.heads) - base : (uint32_t)o.cols;
   const uint32_t e = (uint32_t)x + (uint32_t)o.nq * (t - g * (uint32_t)o.tickets);
   const uint32_t rank = e / cols;
   uint32_t col = e - rank * cols;
