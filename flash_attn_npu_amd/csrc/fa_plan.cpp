@@ -137,25 +137,34 @@ constexpr bool table_fits_lds() {
 }
 static_assert(table_fits_lds(), "LDS budget of one gfx950 CU");
 
-// Default (BLOCK_N, waves) per head dim; BLOCK_M = 32 * waves.
-void default_tiling(int D, int dtype, int *bn, int *nw) {
+// Default (BLOCK_N, waves); BLOCK_M = 32 * waves.
+void default_tiling(const fa_fwd_params *p, int *bn, int *nw) {
+  *nw = 4;
   // fp8 V: 64-key tiles (D = 16: 128), one 32x32x64 MFMA per 64 keys and 32
   // head dims.  16-bit V: 64 keys, except D = 16 (128) and D = 256 (32).
-  // Non-causal D = 128 took the 32-key kernel (three workgroups per CU) before
-  // the 64-key one carried its tile as two 32-key blocks; over grids of 8 to
-  // 1536 tiles and 256 to 8192 keys the 64-key kernel is now the faster on
-  // every one, by 3-9% on full grids and 13-25% up to one tile per CU (fp16,
-  // us, 32 against 64 keys: H16 S2048 43.5 / 37.9, H32 S4096 270 / 258,
-  // H16 S1024 22.9 / 18.3).
-  if (v_is_fp8(dtype))
-    *bn = D == 16 ? 128 : 64;
-  else if (D == 16)
-    *bn = 128;
-  else if (D == 256)
-    *bn = 32;
-  else
-    *bn = 64;
-  *nw = 4;
+  if (v_is_fp8(p->dtype)) {
+    *bn = p->D == 16 ? 128 : 64;
+    return;
+  }
+  *bn = p->D == 16 ? 128 : p->D == 256 ? 32 : 64;
+  if (p->D != 128 || p->causal) return;
+  // Non-causal D = 128: the 64-key kernel (two workgroups per CU, its tile
+  // carried as two 32-key blocks) is 1-10% faster than the 32-key one (three per
+  // CU) on full grids and 8-30% up to one tile per CU (fp16, us, 32 against 64
+  // keys: H16 S2048 44.3 / 37.5, H128 S2048 255 / 250, H16 S1024 23.0 / 18.5).
+  // Timed at 16 to 16384 keys and 1 to 32768 tiles, the 32-key kernel is the faster
+  //  * up to 48 keys, where half of a 64-key tile is padding (H1024 S32 9.8 / 12.4,
+  //    S48 13.5 / 14.6);
+  //  * up to 96 keys on grids of more tiles than the 512 workgroups that the
+  //    64-key kernel has on the chip: a unit is then mostly prologue and
+  //    epilogue, which the third workgroup per CU hides (H1024 S64 15.5 / 16.3,
+  //    S96 20.6 / 23.2).  From 4096 tiles on, eight rounds, it no longer pays
+  //    (H4096 S96 91.5 / 85.7).
+  // At 8192 and 16384 keys with 4096 tiles and more the two are within 2% of each
+  // other, either one ahead from run to run.
+  const int64_t heads = (int64_t)p->B * p->H;  // < 2^62
+  const int64_t tiles = ((int64_t)p->Sq + 127) / 128 * (heads < INT32_MAX ? heads : INT32_MAX);
+  if (p->Sk <= 48 || (p->Sk <= 96 && tiles > 512 && tiles < 4096)) *bn = 32;
 }
 
 int find_kernel(int D, int dtype, int causal, int BN, int NW) {
@@ -183,7 +192,7 @@ constexpr int kDefaultCuCount = 256;
 int make_plan(const fa_fwd_params *p, Plan *out, int cu_count = kDefaultCuCount, int splits = 1) {
   int bn, nw;
   if (p->block_m == 0 && p->block_n == 0) {
-    default_tiling(p->D, p->dtype, &bn, &nw);
+    default_tiling(p, &bn, &nw);
   } else {
     if (p->block_m <= 0 || p->block_n <= 0 || p->block_m % 32 != 0) return FA_ERR_TILING;
     bn = p->block_n;

@@ -12,10 +12,20 @@ from flash_attn_npu_amd import flash_attention_forward as fa
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_default_tile_follows_head_dim(head_dim, block_n, causal, dtype):
-    for n_ctx in (1, 64, 333, 1777, 8192):
+    for n_ctx in (49, 64, 333, 1777, 8192):
         rt = fa._describe_runtime(3, 5, n_ctx, head_dim, causal, dtype=dtype)
         assert rt["tiling_source"] == "fallback"
         assert rt["selected_config"] == {"BLOCK_M": 128, "BLOCK_N": block_n}
+
+
+@pytest.mark.parametrize("heads,n_ctx,block_n", [
+    (3, 1, 32), (3, 48, 32), (3, 49, 64), (2000, 48, 32),    # half a 64-key tile would be padding
+    (512, 96, 64), (513, 96, 32), (513, 49, 32), (513, 97, 64), (257, 129, 64), (4095, 96, 32),
+    (4096, 96, 64), (4096, 48, 32), (64, 16384, 64)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_non_causal_d128_tile_at_its_limits(heads, n_ctx, block_n, dtype):
+    assert fa._query_config(1, heads, n_ctx, 128, False, dtype=dtype)[1] == block_n
+    assert fa._query_config(1, heads, n_ctx, 128, True, dtype=dtype)[1] == 64
 
 
 def _splits(z, h, n_ctx, head_dim, causal):
