@@ -331,6 +331,67 @@ int64_t split_workspace_bytes(const fa_fwd_params *p, int splits) {
   return po >= 0 && b < kMaxWorkspace ? (int64_t)b : -1;
 }
 
+// The split count that is estimated to be the fastest.
+//
+// A grid of at most one tile per CU takes as long as one workgroup needs for all
+// its keys, and splitting them pays what the merge costs: its launch, and one pass
+// of the partial O (tiles * splits of them) out and in.  Both are estimated in
+// us from timings of 1960 shapes with up to 15 split counts each (6 to 320
+// tiles, 300 to 16384 keys, every head dim, fp16, bf16 and e5m2 V):
+//  * 5 us and a time per key that grows with D (H16 S1024 D128: 18.5 us, H8 S2048
+//    29.4, H1 S4096 D16 31);
+//  * the merge: 4.5 us, 0.2 per split and 0.03 per tile and split at D = 128
+//    (0.6 of it where causal, as fitted: both masks store every partial O);
+//  * a split call takes the host about 14.5 us, whatever its size.
+// Tried are the powers of two and the counts that fill the CUs, in runs of at
+// least 128 keys, none of them empty (H1 S10240 D32, 80 tiles: 36.5 us at 3
+// splits, 47.1 at 2), on at most
+//  * one workgroup per CU;
+//  * causal, where half of the work is missing: 288 workgroups (H2 S6144 D128, 96
+//    tiles: 39 us at 3 splits, 48 at 2), at D = 256 from runs of 1365 keys on (H2
+//    S6144 74 / 87); 512 at D <= 128 with up to 128 tiles and such runs (H1 S16384
+//    D128: 101 us at 4, 124 at 2); 384 for two runs of 2048 keys (H3 S6144 D256,
+//    144 tiles: 99 us, 143 unsplit), not more (H4 S8192 D256, 256 tiles: 235 / 204).
+// The picks are 2.2% slower than the fastest count on average.  Against the rule
+// of 64K key-columns a run and one workgroup per CU, two if causal, 8.4% slower
+// on average, they are up to 2.3x faster, and 3-7% slower on 16 of the shapes (15%
+// on one between them: H1 S14000 D16 causal).
+int choose_kv_splits(const fa_fwd_params *p) {
+  // Shape-only (no pointer or stride checks): usable before tensors exist.
+  if (p == nullptr || p->B <= 0 || p->H <= 0 || p->Sq <= 0 || p->Sk <= 0) return 1;
+  if (!is_supported_head_dim(p->D) || !is_valid_dtype(p->dtype)) return 1;
+  Plan plan;
+  if (make_plan(p, &plan) != FA_OK || !kKernelMeta[plan.kernel].splittable) return 1;
+  const int64_t tiles = plan.total_tiles, D = p->D;
+  if (tiles > kDefaultCuCount) return 1;
+  const int64_t kv_tiles = ((int64_t)p->Sk + plan.BN - 1) / plan.BN;
+  const int64_t keys = p->Sk;
+  const double key_us = (D == 16 ? 6.5 : D == 32 ? 7.5 : D == 64 ? 9.3 : D == 128 ? 11.7 : 23.0) / 1024;
+  const double unit_us = 0.030 * (p->causal ? 0.6 : 1.0) * D / 128;
+  double best = 0.0;
+  int splits = 1;
+  for (int s = 2; s <= kMaxKvSplits && p->Sk / s >= 128; ++s) {
+    const int64_t run_tiles = (kv_tiles + s - 1) / s, units = tiles * s;
+    if ((kv_tiles + run_tiles - 1) / run_tiles < s) continue;  // empty runs at the end
+    const int64_t run = run_tiles * plan.BN < keys ? run_tiles * plan.BN : keys;
+    int64_t fill = kDefaultCuCount;
+    if (p->causal && (D <= 128 || run >= 1365)) fill = 288;
+    if ((s & (s - 1)) != 0 && s != kDefaultCuCount / tiles && s != fill / tiles) continue;
+    int64_t limit = fill;
+    if (p->causal && D <= 128 && tiles <= 128 && run >= 1365) limit = 512;
+    if (p->causal && s == 2 && run >= 2048 && limit < 384) limit = 384;
+    if (units > limit) continue;
+    double split_us = run * key_us + 4.5 + 0.2 * s + unit_us * (double)units;
+    if (split_us < 14.5 - 5.0) split_us = 14.5 - 5.0;
+    const double gain = keys * key_us - split_us;
+    if (gain > best) {
+      best = gain;
+      splits = s;
+    }
+  }
+  return splits;
+}
+
 }  // namespace
 
 #ifndef FA_SOURCE_HASH
@@ -452,48 +513,6 @@ int64_t fa_split_workspace_bytes(const fa_fwd_params *p, int32_t kv_splits) {
   return bytes >= 0 ? bytes : (int64_t)FA_ERR_SHAPE;
 }
 
-int32_t fa_default_kv_splits(const fa_fwd_params *p) {
-  // Shape-only (no pointer or stride checks): usable before tensors exist.
-  if (p == nullptr || p->B <= 0 || p->H <= 0 || p->Sq <= 0 || p->Sk <= 0) return 1;
-  if (!is_supported_head_dim(p->D) || !is_valid_dtype(p->dtype)) return 1;
-  Plan plan;
-  if (make_plan(p, &plan) != FA_OK) return 1;
-  const KernelMeta &e = kKernelMeta[plan.kernel];
-  if (!e.splittable) return 1;
-  // A grid of at most one tile per CU takes as long as one workgroup needs
-  // for all its keys, and splitting them pays what the merge costs: its launch,
-  // and one pass of the partial O (tiles * splits of them) out and in.  Both are
-  // estimated in us from timings over 8 to 256 tiles, 256 to 8192 keys and
-  // every head dim (fp16, 2 to 16 splits); the power of two with the
-  // largest gain wins, or none:
-  //  * a lone workgroup's time per key grows with D (H16 S1024 D128: 18.3 us,
-  //    H8 S2048 29.6, H4 S4096 31.5 at D = 16);
-  //  * the merge costs 5 us, 0.2 per split and 0.03 per tile and split at
-  //    D = 128; causal launches write less, their runs past the diagonal being empty;
-  //  * runs of at least 128 keys, and one workgroup per CU: more only when
-  //    causal, where half of the work is missing, with runs of 2048 keys.
-  // Against the rule before (at least 64K key-columns a run, one workgroup per
-  // CU, two if causal), us: H8 S2048 D16 18.2 -> 15.5, H1 S4096 D32 23.4 ->
-  // 16.6, H2 S2048 D64 18.0 -> 16.4, H16 S1024 D128 26.2 -> 18.3, H16 S1024
-  // D256 causal 51.9 -> 31.2; over that sweep it is within 1% of the fastest
-  // choice on average (3.6% before).
-  if (plan.total_tiles > kDefaultCuCount) return 1;
-  const double key_us = (p->D == 16 ? 6.5 : p->D == 32 ? 7.5 : p->D == 64 ? 9.3 : p->D == 128 ? 11.7 : 23.0) / 1024;
-  const double tile_us = 0.030 * (p->causal ? 0.6 : 1.0) * p->D / 128;
-  double best = 0.0;
-  int splits = 1;
-  for (int s = 2; s <= kMaxKvSplits; s *= 2) {
-    const int64_t run = p->Sk / s, groups = plan.total_tiles * s;
-    int64_t limit = kDefaultCuCount;
-    if (p->causal && run >= 2048) limit = plan.total_tiles <= kDefaultCuCount / 2 && p->D <= 128 ? 512 : 384;
-    if (run < 128 || groups > limit) break;
-    const double gain = p->Sk * key_us * (1.0 - 1.0 / s) - (5.0 + 0.2 * s + tile_us * (double)groups);
-    if (gain > best) {
-      best = gain;
-      splits = s;
-    }
-  }
-  return splits;
-}
+int32_t fa_default_kv_splits(const fa_fwd_params *p) { return choose_kv_splits(p); }
 
 }  // extern "C"

@@ -147,3 +147,16 @@ def test_split_graph_replays(fa, monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want_o) and torch.equal(lse, want_l), rep
+
+
+@pytest.mark.parametrize("shape,causal,splits", [((1, 1, 10240, 32), False, 3), ((1, 5, 4096, 256), True, 2),
+                                                 ((2, 3, 1500, 16), False, None)])
+def test_default_splits_of_odd_tile_counts(fa, shape, causal, splits):
+    """The library's own count between powers of two, and where the partial results exceed the static buffer."""
+    rt = fa._describe_runtime(*shape, causal)
+    assert splits is None or rt["kv_splits"] == splits
+    q, k, v = _inputs(47, shape, torch.float16)
+    out, lse = fa.attention(q, k, v, causal, 0.1, return_lse=True)
+    o64, l64 = attention_fp64(q, k, v, causal, 0.1, heads_per_chunk=2)
+    assert (out.float() - o64.half().float()).abs().max().item() <= 5e-3
+    assert (lse.double() - l64).abs().max().item() <= 1e-3

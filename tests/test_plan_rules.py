@@ -36,7 +36,7 @@ def test_split_choice_at_its_limits():
     # 128 tiles of 1024 keys: the merge would cost more than the halved runs save.
     assert _splits(1, 16, 1024, 128, False) == 1
     assert _splits(1, 16, 1024, 256, True) == 1
-    # 128 tiles of 4096 keys: two runs fill the CUs.
+    # 128 tiles of 4096 and 2048 keys: two runs fill the CUs.
     assert _splits(1, 4, 4096, 128, False) == 2
     assert _splits(1, 8, 2048, 16, False) == 2
     # One tile per CU and more: none.
@@ -51,3 +51,22 @@ def test_split_choice_at_its_limits():
     for n_ctx in (129, 300, 1000, 4097, 100000):
         s = _splits(1, 1, n_ctx, 128, False)
         assert s == 1 or (n_ctx // s >= 128 and s * -(-n_ctx // 128) <= 256)
+
+
+@pytest.mark.parametrize("head_dim", [32, 64, 128, 256])
+def test_splits_fill_the_cus_between_powers_of_two(head_dim):
+    # 80 tiles: 3 runs make 240 workgroups, 2 only 160; 40 and 48 tiles: 6 and 5.
+    assert _splits(1, 1, 10240, head_dim, False) == 3
+    assert _splits(1, 1, 5120, head_dim, False) in (4, 6)
+    assert _splits(1, 1, 6144, head_dim, False) in (4, 5)
+    # Causal, 96 tiles: 288 workgroups.
+    assert _splits(1, 2, 6144, head_dim, True) in (3, 4)
+
+
+def test_no_split_leaves_empty_runs():
+    for head_dim, bn in ((16, 128), (64, 64), (128, 64), (256, 32)):
+        for n_ctx in (1000, 1500, 2177, 3000, 4097, 5000, 8193, 8200, 10000):
+            for heads in (1, 2, 3):
+                s = _splits(1, heads, n_ctx, head_dim, False)
+                kv_tiles = -(-n_ctx // bn)
+                assert -(-kv_tiles // -(-kv_tiles // s)) == s, (head_dim, n_ctx, heads, s)
