@@ -1,7 +1,7 @@
 // fa_plan.cpp -- host-only half of libfa_mi355x.so: the kernel table's
 // metadata, tile planning and the C-ABI calls that make no HIP call
 // (fa_validate, fa_query_config, fa_default_kv_splits,
-// fa_split_workspace_bytes, fa_kernel_info, fa_kernel_wg_per_cu, ...).
+// fa_workspace_kv_splits, fa_split_workspace_bytes, fa_kernel_info, fa_kernel_wg_per_cu, ...).
 //
 // Plain C++17 with no HIP header: fa_fwd.hip includes this file (the library
 // stays one translation unit, and the kernel pointer table there is built
@@ -331,7 +331,8 @@ int64_t split_workspace_bytes(const fa_fwd_params *p, int splits) {
   return po >= 0 && b < kMaxWorkspace ? (int64_t)b : -1;
 }
 
-// The split count that is estimated to be the fastest.
+// The split count that is estimated to be the fastest; with any_workspace false,
+// of those that fa_default_kv_splits may return.
 //
 // A grid of at most one tile per CU takes as long as one workgroup needs for all
 // its keys, and splitting them pays what the merge costs: its launch, and one pass
@@ -356,7 +357,7 @@ int64_t split_workspace_bytes(const fa_fwd_params *p, int splits) {
 // of 64K key-columns a run and one workgroup per CU, two if causal, 8.4% slower
 // on average, they are up to 2.3x faster, and 3-7% slower on 16 of the shapes (15%
 // on one between them: H1 S14000 D16 causal).
-int choose_kv_splits(const fa_fwd_params *p) {
+int choose_kv_splits(const fa_fwd_params *p, bool any_workspace) {
   // Shape-only (no pointer or stride checks): usable before tensors exist.
   if (p == nullptr || p->B <= 0 || p->H <= 0 || p->Sq <= 0 || p->Sk <= 0) return 1;
   if (!is_supported_head_dim(p->D) || !is_valid_dtype(p->dtype)) return 1;
@@ -381,6 +382,12 @@ int choose_kv_splits(const fa_fwd_params *p) {
     if (p->causal && D <= 128 && tiles <= 128 && run >= 1365) limit = 512;
     if (p->causal && s == 2 && run >= 2048 && limit < 384) limit = 384;
     if (units > limit) continue;
+    // Callers of fa_fwd_split_static ask fa_default_kv_splits for their count: what
+    // its buffer cannot hold is theirs only where runs keep 64K key-columns.
+    if (!any_workspace && (tiles > 128 || s * (int64_t)65536 > p->Sk * D)) {
+      const int64_t bytes = split_workspace_bytes(p, s);
+      if (bytes < 0 || bytes > (int64_t)FA_STATIC_SCRATCH_BYTES) continue;
+    }
     double split_us = run * key_us + 4.5 + 0.2 * s + unit_us * (double)units;
     if (split_us < 14.5 - 5.0) split_us = 14.5 - 5.0;
     const double gain = keys * key_us - split_us;
@@ -513,6 +520,8 @@ int64_t fa_split_workspace_bytes(const fa_fwd_params *p, int32_t kv_splits) {
   return bytes >= 0 ? bytes : (int64_t)FA_ERR_SHAPE;
 }
 
-int32_t fa_default_kv_splits(const fa_fwd_params *p) { return choose_kv_splits(p); }
+int32_t fa_default_kv_splits(const fa_fwd_params *p) { return choose_kv_splits(p, false); }
+
+int32_t fa_workspace_kv_splits(const fa_fwd_params *p) { return choose_kv_splits(p, true); }
 
 }  // extern "C"

@@ -37,7 +37,7 @@ RESULT_DIR_NAME = "result_dir"
 # way every workgroup walks its share of the balanced tile schedule (the
 # reference's persistent grid, flash_attention_forward.py:24,616-623).
 DEFAULT_PERSISTENT_PROGRAMS = 0
-# 0 = the library's split-KV choice (fa_default_kv_splits: only grids of at
+# 0 = the library's split-KV choice (fa_workspace_kv_splits: only grids of at
 # most one tile per CU, where the shorter runs save more than the merge costs);
 # KV_SPLITS in [1, 64] overrides.
 DEFAULT_KV_SPLITS = 0
@@ -231,6 +231,8 @@ def _load_library():
     lib.fa_fwd_split_static.restype = ctypes.c_int
     lib.fa_default_kv_splits.argtypes = [P]
     lib.fa_default_kv_splits.restype = ctypes.c_int32
+    lib.fa_workspace_kv_splits.argtypes = [P]
+    lib.fa_workspace_kv_splits.restype = ctypes.c_int32
     if lib.fa_params_size() != ctypes.sizeof(FaFwdParams):
         raise RuntimeError("fa_fwd_params layout mismatch between the library and this binding")
     _LIB = lib
@@ -372,7 +374,7 @@ def _describe_runtime(z, h, n_ctx, head_dim, causal, bm=None, bn=None, dtype=tor
     cfg = list(out)
     splits = _get_kv_splits()
     if splits == 0:
-        splits = int(lib.fa_default_kv_splits(ctypes.byref(p)))
+        splits = int(lib.fa_workspace_kv_splits(ctypes.byref(p)))
     return {
         "selected_config": {"BLOCK_M": cfg[0], "BLOCK_N": cfg[1]},
         "tiling_source": tiling_source,
@@ -466,7 +468,7 @@ def _launch_plan(lib, q, k, v, out, causal, bm, bn, programs, split_env):
     p.causal = 1 if causal else 0
     p.block_m, p.block_n = int(bm), int(bn)
     p.num_programs = programs
-    splits = split_env if split_env else int(lib.fa_default_kv_splits(ctypes.byref(p)))
+    splits = split_env if split_env else int(lib.fa_workspace_kv_splits(ctypes.byref(p)))
     nbytes = 0
     if splits > 1:
         nbytes = int(lib.fa_split_workspace_bytes(ctypes.byref(p), splits))

@@ -180,8 +180,13 @@ int fa_fwd_split(const fa_fwd_params *p, int32_t kv_splits, void *workspace, int
 
 /* The library's split choice for these parameters: > 1 only when the unsplit
  * grid has at most one (head, m-tile) tile per CU and the shorter runs are
- * estimated to save more than the merge costs.  Host-only. */
+ * estimated to save more than the merge costs.  fa_workspace_kv_splits is the
+ * choice where any workspace can be had; fa_default_kv_splits leaves out
+ * counts whose partial results exceed FA_STATIC_SCRATCH_BYTES, unless the grid
+ * has at most one tile per two CUs and every run 65536 key-columns (Sk / splits
+ * * D).  Host-only. */
 int32_t fa_default_kv_splits(const fa_fwd_params *p);
+int32_t fa_workspace_kv_splits(const fa_fwd_params *p);
 
 /* ---- No-allocation split-KV.  No counterpart in the reference.  For callers
  * that cannot allocate device memory (code under HIP graph capture, tight

@@ -2,7 +2,7 @@
 // flash_attn_npu_amd/csrc/fa_plan.cpp under AddressSanitizer and
 // UndefinedBehaviorSanitizer by tests/test_host_sanitizers.py (no HIP, no GPU).
 //
-// It walks fa_validate, fa_query_config, fa_default_kv_splits,
+// It walks fa_validate, fa_query_config, fa_default_kv_splits, fa_workspace_kv_splits,
 // fa_split_workspace_bytes, fa_kernel_info, fa_kernel_wg_per_cu and
 // fa_error_string over hand-picked edge cases and a seeded random sweep
 // (sizes and strides up to their type limits, negative values, NULL
@@ -118,6 +118,8 @@ static void check_params(const fa_fwd_params &p, const KernelRow *rows, int nk) 
   }
   const int32_t splits = fa_default_kv_splits(&p);
   CHECK(splits >= 1 && splits <= 64, "default splits %d", splits);
+  const int32_t any_splits = fa_workspace_kv_splits(&p);
+  CHECK(any_splits >= 1 && any_splits <= 64, "workspace splits %d", any_splits);
   int64_t prev = 0;
   for (int32_t s = 0; s <= 66; s += (s < 4 ? 1 : 31)) {
     const int64_t b = fa_split_workspace_bytes(&p, s);
@@ -161,6 +163,7 @@ int main() {
   int32_t cfg[FA_CFG_COUNT];
   CHECK(fa_query_config(nullptr, cfg) == FA_ERR_NULL, "query(NULL)");
   CHECK(fa_default_kv_splits(nullptr) == 1, "splits(NULL)");
+  CHECK(fa_workspace_kv_splits(nullptr) == 1, "workspace splits(NULL)");
   CHECK(fa_split_workspace_bytes(nullptr, 2) == FA_ERR_NULL, "workspace(NULL)");
 
   // Every kernel of the table, at the benchmark sizes and at ragged ones.

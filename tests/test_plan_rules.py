@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -61,6 +63,33 @@ def test_splits_fill_the_cus_between_powers_of_two(head_dim):
     assert _splits(1, 1, 6144, head_dim, False) in (4, 5)
     # Causal, 96 tiles: 288 workgroups.
     assert _splits(1, 2, 6144, head_dim, True) in (3, 4)
+
+
+def _choices(z, h, s_q, s_k, head_dim, causal, programs=0):
+    lib = fa._load_library()
+    p = fa._shape_params(z, h, s_q, head_dim, causal, programs=programs)
+    p.Sk = s_k
+    splits = [f(ctypes.byref(p)) for f in (lib.fa_default_kv_splits, lib.fa_workspace_kv_splits)]
+    return splits, [lib.fa_split_workspace_bytes(ctypes.byref(p), s) for s in splits]
+
+
+def test_default_choice_fits_the_static_buffer():
+    """What fa_default_kv_splits returns can be passed to fa_fwd_split_static, but for long
+    runs on grids of at most one tile per two CUs."""
+    larger = 0
+    for head_dim in (16, 64, 128, 256):
+        for heads in range(1, 14):
+            for n_ctx in (1024, 1500, 2048, 3000, 4096, 5000, 8192, 16384):
+                for causal in (False, True):
+                    tiles = heads * -(-n_ctx // 128)
+                    (default, any_ws), (nbytes, _) = _choices(1, heads, n_ctx, n_ctx, head_dim, causal)
+                    assert default <= 1 or nbytes <= 32 << 20 or (
+                        tiles <= 128 and default * 65536 <= n_ctx * head_dim), (head_dim, heads, n_ctx, causal)
+                    larger += any_ws != default
+    assert larger > 0
+    # 160 tiles, 40 MiB of partial results: only where a workspace can be had.
+    assert _choices(1, 5, 4096, 4096, 256, True)[0] == [1, 2]
+    assert _splits(1, 5, 4096, 256, True) == 2
 
 
 def test_no_split_leaves_empty_runs():
