@@ -360,15 +360,18 @@ int64_t split_workspace_bytes(const fa_fwd_params *p, int splits) {
 int choose_kv_splits(const fa_fwd_params *p, bool any_workspace) {
   // Shape-only (no pointer or stride checks): usable before tensors exist.
   if (p == nullptr || p->B <= 0 || p->H <= 0 || p->Sq <= 0 || p->Sk <= 0) return 1;
-  if (!is_supported_head_dim(p->D) || !is_valid_dtype(p->dtype)) return 1;
+  if (!is_supported_head_dim(p->D) || !is_valid_dtype(p->dtype) || p->num_programs < 0) return 1;
   Plan plan;
   if (make_plan(p, &plan) != FA_OK || !kKernelMeta[plan.kernel].splittable) return 1;
   const int64_t tiles = plan.total_tiles, D = p->D;
   if (tiles > kDefaultCuCount) return 1;
   const int64_t kv_tiles = ((int64_t)p->Sk + plan.BN - 1) / plan.BN;
-  const int64_t keys = p->Sk;
+  const int64_t keys = p->causal && p->Sq < p->Sk ? p->Sq : p->Sk;  // of the longest m-tile
   const double key_us = (D == 16 ? 6.5 : D == 32 ? 7.5 : D == 64 ? 9.3 : D == 128 ? 11.7 : 23.0) / 1024;
   const double unit_us = 0.030 * (p->causal ? 0.6 : 1.0) * D / 128;
+  // A program count below the tiles makes each program walk several units anyway.
+  const int64_t programs = p->num_programs > 0 && p->num_programs < tiles ? p->num_programs : 0;
+  auto rounds = [&](int64_t units) { return programs > 0 ? (double)((units + programs - 1) / programs) : 1.0; };
   double best = 0.0;
   int splits = 1;
   for (int s = 2; s <= kMaxKvSplits && p->Sk / s >= 128; ++s) {
@@ -388,9 +391,9 @@ int choose_kv_splits(const fa_fwd_params *p, bool any_workspace) {
       const int64_t bytes = split_workspace_bytes(p, s);
       if (bytes < 0 || bytes > (int64_t)FA_STATIC_SCRATCH_BYTES) continue;
     }
-    double split_us = run * key_us + 4.5 + 0.2 * s + unit_us * (double)units;
+    double split_us = run * key_us * rounds(units) + 4.5 + 0.2 * s + unit_us * (double)units;
     if (split_us < 14.5 - 5.0) split_us = 14.5 - 5.0;
-    const double gain = keys * key_us - split_us;
+    const double gain = keys * key_us * rounds(tiles) - split_us;
     if (gain > best) {
       best = gain;
       splits = s;

@@ -99,3 +99,14 @@ def test_no_split_leaves_empty_runs():
                 s = _splits(1, heads, n_ctx, head_dim, False)
                 kv_tiles = -(-n_ctx // bn)
                 assert -(-kv_tiles // -(-kv_tiles // s)) == s, (head_dim, n_ctx, heads, s)
+
+
+def test_splits_count_visible_keys_and_programs():
+    # Causal with more keys than queries: only Sq keys are ever visible.
+    for heads in (8, 100, 192):
+        assert _choices(1, heads, 128, 8192, 64, True)[0] == [1, 1]
+    # Fewer programs than tiles: splitting them shortens nothing.
+    assert _choices(1, 3, 8192, 8192, 64, True)[0] == [2, 2]
+    assert _choices(1, 3, 8192, 8192, 64, True, programs=64)[0] == [1, 1]
+    assert _choices(1, 1, 4096, 4096, 128, False, programs=16)[0] == [1, 1]
+    assert _choices(1, 1, 4096, 4096, 128, False, programs=256)[0] == [8, 8]
