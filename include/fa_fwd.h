@@ -96,10 +96,10 @@ typedef struct fa_fwd_params {
   int32_t dtype;              /* enum fa_dtype; o has the type of q and k */
   int32_t causal;             /* 0 or 1 */
   float sm_scale;
-  int32_t block_m;            /* 0 = library default for (D, dtype, causal, S) */
+  int32_t block_m;            /* 0 = library default for the shape, dtype and mask */
   int32_t block_n;            /* 0 = library default; must be given with block_m */
-  int32_t num_programs;       /* 0 = one workgroup per tile; >0 = persistent grid
-                                 capped at this many workgroups (the reference's
+  int32_t num_programs;       /* 0 = as many workgroups as are resident at once;
+                                 >0 = at most this many (the reference's
                                  PERSISTENT_PROGRAMS, flash_attention_forward.py:616-623) */
 } fa_fwd_params;
 
