@@ -151,8 +151,8 @@ def _check_resources(remarks, table):
         name, res = by_key[_entry_key(table[i])]
         assert res["ScratchSize [bytes/lane]"] == 0 and res["VGPRs Spill"] == 0, \
             f"default kernel {i} ({name}) spills: {res}"
-        # Scalars kept live through a unit push the tile loop's own into vector lanes: 128 here
-        # (103 now) made every launch 1-2% slower.
+        # Scalars kept live through a unit push the tile loop's own into vector lanes: the e5m2 D = 64
+        # kernel with 115 of them instead of 57 took 134 us for B4 H32 S2048 instead of 123.
         assert res["SGPRs Spill"] <= 108, f"default kernel {i} ({name}) spills {res['SGPRs Spill']} scalars"
     merge = [res for name, res in remarks.items() if "fa_merge_kernel" in name]
     assert len(merge) == 2 and all(r["ScratchSize [bytes/lane]"] == 0 for r in merge)
